@@ -36,11 +36,11 @@ def _hipcc() -> str:
     raise RuntimeError("hipcc not found (set HIPCC or install ROCm)")
 
 
-HIP_SOURCES = ("dk_api.hip", "dk_paging.hip", "dk_append.hip")
-# pass-1 kernel tables: each compiled once per head_dim (-DDK_HEAD_DIM=...)
+HIP_SOURCES = ("dk_api.hip", "dk_paging.hip", "dk_append.hip", "dk_extend_api.hip")
+# pass-1 and extend kernel tables: each compiled once per head_dim (-DDK_HEAD_DIM=...)
 KERNEL_SOURCES = ("dk_f16.hip", "dk_bf16.hip", "dk_f16_mfma.hip", "dk_bf16_mfma.hip",
                   "dk_f16_kv8.hip", "dk_bf16_kv8.hip", "dk_f16_kv8_mfma.hip",
-                  "dk_bf16_kv8_mfma.hip")
+                  "dk_bf16_kv8_mfma.hip", "dk_extend.hip")
 HEAD_DIMS = (64, 128, 256)
 
 

@@ -47,6 +47,11 @@ class DkStrides(ctypes.Structure):
                 ("q_b", "q_h", "kv_p", "kv_r", "kv_s", "kv_h", "o_b", "o_h")]
 
 
+class DkExtendStrides(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int64) for n in
+                ("q_b", "q_h", "k_s", "k_h", "v_s", "v_h", "o_b", "o_h")]
+
+
 class DkOptions(ctypes.Structure):
     _fields_ = [("qk_path", ctypes.c_int32), ("waves_per_group", ctypes.c_int32),
                 ("waves_per_cu", ctypes.c_int32), ("schedule", ctypes.c_int32),
@@ -98,6 +103,11 @@ SIGNATURES = {
                                         _I32, _I32, _I32, _I32, _I32, _I32, _I64, _I64, _I32,
                                         ctypes.c_float, ctypes.c_float,
                                         ctypes.POINTER(DkStrides), _P]),
+    "dk_extend_attention": (ctypes.c_int, [_P, _P, _P, _P, _I64, _I64, ctypes.POINTER(_I32),
+                                           ctypes.POINTER(_I32), ctypes.POINTER(_I32), _P, _I32,
+                                           _I64, _I32, _I32, _I32, _I64, _I32, _I32,
+                                           ctypes.POINTER(DkExtendStrides), ctypes.c_float,
+                                           ctypes.c_float, ctypes.c_float, _I32, _P, _P]),
     "dk_decode_partials": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _SZ, _I32, _I32, _I32, _I32,
                                           _I32, _I64, _I64, _I32, ctypes.POINTER(DkStrides),
                                           _I32, ctypes.POINTER(DkOptions), _P]),

@@ -1,7 +1,7 @@
 """SGLang attention backend on the MI355X split-KV decode kernel.
 
 Counterpart of the reference adapter (integration/sglang_backend.py:50-137): decode steps
-go to the HIP kernel through `decode_attention`; prefill (extend) stays outside this path.
+go to the HIP kernel through `decode_attention`, prefill (extend) to `extend.extend_attention`.
 Two entry styles are provided:
 
 * SGLang's backend API — `init_forward_metadata(forward_batch)` once per batch, then
@@ -39,6 +39,7 @@ from typing import Optional
 import torch
 
 import attention
+import extend
 import paging
 from attention import decode_attention
 
@@ -92,7 +93,7 @@ class DecodeMetadata:
 
 
 class SplitKVHipBackend(_backend_base()):
-    """Decode attention on the HIP split-KV kernel; prefill on PyTorch SDPA."""
+    """Decode attention on the HIP split-KV kernel; prefill on the HIP extend kernel."""
 
     def __init__(self, model_runner=None, split_kv: Optional[int] = None):
         self.model_runner = model_runner
@@ -203,10 +204,13 @@ class SplitKVHipBackend(_backend_base()):
     def forward_extend(self, q, k, v, layer, forward_batch, save_kv_cache: bool = True,
                        **kwargs):
         """Prefill / extend: causal attention of the new tokens over each request's cached
-        prefix and themselves, with PyTorch SDPA per request (outside the decode path)."""
+        prefix and themselves: one launch of the extend kernel for the calls that it takes
+        (extend.takes), else PyTorch SDPA per request."""
         sinks = self._sinks(kwargs.pop("sinks", None), layer)
         _refuse_extras("forward_extend", kwargs)
         pool = forward_batch.token_to_kv_pool
+        # the one device read of the call, before the work that it would wait for
+        row_ids = forward_batch.req_pool_indices.tolist()
         if k is not None and save_kv_cache:
             self._save(pool, layer, forward_batch.out_cache_loc, k, v)
         hq, hkv, d = layer.tp_q_head_num, layer.tp_k_head_num, layer.head_dim
@@ -217,10 +221,18 @@ class SplitKVHipBackend(_backend_base()):
         out = torch.empty_like(qv)
         ext = forward_batch.extend_seq_lens_cpu
         lens = forward_batch.seq_lens_cpu
-        rows = forward_batch.req_pool_indices.tolist()
+        reqs = [(row, int(n_new), int(n_all)) for row, n_new, n_all in
+                zip(row_ids, list(ext), list(lens))]
+        rows, new_lens, all_lens = zip(*reqs) if reqs else ((), (), ())
+        scale, cap, win = _scale(layer, d) or 1.0 / math.sqrt(d), _logit_cap(layer), _window(layer)
+        if (hq, hkv, d) == (qv.shape[1], kb.shape[1], kb.shape[2]) and \
+                extend.takes(qv, kb, vb, req_to_token, rows, new_lens, all_lens, scale, cap, ks,
+                             vs, sinks):
+            extend.extend_attention(qv, kb, vb, req_to_token, rows, new_lens, all_lens, out,
+                                    scale, cap, win, ks, vs, sinks)
+            return out.view(-1, hq * d)
         start = 0
-        for row, n_new, n_all in zip(rows, list(ext), list(lens)):
-            n_new, n_all = int(n_new), int(n_all)
+        for row, n_new, n_all in reqs:
             slots = req_to_token[row, :n_all].long()
             kk = kb[slots].float().transpose(0, 1) * ks      # (hkv, n_all, d)
             vv = vb[slots].float().transpose(0, 1) * vs
@@ -232,11 +244,8 @@ class SplitKVHipBackend(_backend_base()):
             pos_q = torch.arange(n_all - n_new, n_all, device=q.device)[:, None]
             kpos = torch.arange(n_all, device=q.device)[None, :]
             mask = kpos <= pos_q
-            win = _window(layer)
             if win:                                   # sliding window: the last `win` keys
                 mask &= kpos > pos_q - win
-            scale = _scale(layer, d) or 1.0 / math.sqrt(d)
-            cap = _logit_cap(layer)
             if cap or sinks is not None:
                 # soft-capped scores or attention sinks: SDPA has neither, so attend
                 # explicitly (a sink is one more logit per head, with no value)

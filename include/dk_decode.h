@@ -319,6 +319,34 @@ int dk_append_kv_fp8(void* q, const void* k_new, const void* v_new, int64_t new_
                      int64_t num_indices, int32_t dtype, float k_scale, float v_scale,
                      const dk_strides* strides, void* hip_stream);
 
+/* Element strides of dk_extend_attention: q / out rows (one per new token) and heads, K and V
+ * pool token slots and kv heads; the head_dim stride is 1 everywhere. */
+typedef struct dk_extend_strides {
+  int64_t q_b, q_h, k_s, k_h, v_s, v_h, o_b, o_h;
+} dk_extend_strides;
+
+/* Extend (prefill) attention over a token pool: request b's new_lens[b] new tokens are the
+ * last of its all_lens[b] tokens; new token i (position p = all_lens[b] - new_lens[b] + i)
+ * attends to positions <= p (with window > 0, to the last `window` of them), whose K and V
+ * rows are pool slots req_to_token[rows[b]][position] (a negative slot counts from the pool's
+ * end; a slot outside the pool gives NaN to the tokens that attend to it). q and out hold
+ * (num_tokens, num_q_heads, head_dim): the requests' new tokens one request after another.
+ * k_pool / v_pool hold (num_slots, num_kv_heads, head_dim) of q's type or fp8 (kv_dtype).
+ * Scores are q.k * score_scale (> 0; for an fp8 pool it includes K's scale), soft-capped when
+ * logit_cap != 0; the output is scaled by v_scale; sinks as in dk_options. rows, new_lens and
+ * all_lens are HOST arrays of `batch` entries, read before the call returns; the rest is
+ * device memory, used on hip_stream. req_to_token rows are req_stride entries apart,
+ * num_rows of them. The SGLang prefill path (the reference leaves it to other libraries,
+ * integration/sglang_backend.py:94-99). */
+int dk_extend_attention(const void* q, const void* k_pool, const void* v_pool,
+                        const int32_t* req_to_token, int64_t req_stride, int64_t num_rows,
+                        const int32_t* rows, const int32_t* new_lens, const int32_t* all_lens,
+                        void* out, int32_t batch, int64_t num_tokens, int32_t num_q_heads,
+                        int32_t num_kv_heads, int32_t head_dim, int64_t num_slots, int32_t dtype,
+                        int32_t kv_dtype, const dk_extend_strides* strides, float score_scale,
+                        float v_scale, float logit_cap, int32_t window, const float* sinks,
+                        void* hip_stream);
+
 /* Pass 1 only: writes partial_O / partial_m / partial_l for split_kv >= 1 splits into
  * the workspace (layout from dk_partials_layout; partial_m is the split's max of
  * q.k*scale, -1e9 for an empty split, partial_l = sum exp(score - partial_m),
