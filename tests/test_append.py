@@ -186,3 +186,30 @@ def test_fp8_append_then_decode_matches_oracle():
                                          to_np(ids), to_np(last))
     err = np.abs(out.float().cpu().numpy() - want).max()
     assert err <= 1e-2, err
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(1, 1, 2), (9, 3, 6), (5, 5, 64), (28, 4, 66), (4, 1, 256),
+                                      (13, 1, 96)])
+@pytest.mark.parametrize("style", [0, 1])
+@pytest.mark.parametrize("layout_", ["plain", "fused", "unaligned"])
+def test_append_sizes_and_alignments(hq, hkv, d, style, layout_):
+    # head counts around a thread's 4 heads, head dims with and without whole vectors, rows of a
+    # fused projection (strided), and rows that are no multiple of 4 bytes apart from aligned
+    dtype = torch.float16
+    lens = [1, 16, 0, 33, 700]
+    print(f"[case] append {hq}/{hkv}/{d} style={style} {layout_}", flush=True)
+    q, kv, indptr, ids, last, k_new, v_new = _inputs(dtype, lens, hq, hkv, d, seed=d + style)
+    if layout_ != "plain":
+        n, w = len(lens), hq + 2 * hkv
+        off = 1 if layout_ == "unaligned" else 0
+        buf = torch.empty(n * w * d + off, dtype=dtype, device=DEV)[off:].view(n, w, d)
+        buf.copy_(torch.cat([q, k_new, v_new], dim=1))
+        q, k_new, v_new = buf.split([hq, hkv, hkv], dim=1)
+    inv = paging.rope_inv_freq(d)
+    want_kv, want_q = oapp.append_kv(to_np(kv), to_np(q), to_np(k_new), to_np(v_new),
+                                     to_np(indptr), to_np(ids), to_np(last),
+                                     inv_freq=to_np(inv), style=style)
+    paging.append_kv(q, k_new, v_new, kv, indptr, ids, last, inv_freq=inv, rope_style=style)
+    torch.cuda.synchronize()
+    _close(kv, want_kv, dtype)
+    _close(q, want_q, dtype)
