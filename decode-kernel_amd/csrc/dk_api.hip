@@ -344,6 +344,22 @@ int auto_split_fill(const Problem& p, const Plan& pl, int cus, size_t ws_bytes) 
   return total <= ws_bytes ? (int)s : 0;
 }
 
+// Whether the balanced schedule runs its build for long segments (kLongSegmentPages): one kv
+// head per workgroup, 16-bit rows at D = 128 with 3 or 4 q heads per kv head (VALU q.k path),
+// default wave counts of at most 2 per workgroup, and a mean segment long enough: ranges +
+// batch segments, or, where the ranges of a uniform batch (plan hint) start and end with its
+// sequences, the larger of the two.
+bool long_segments(const Problem& p, const Plan& pl, int hp, int64_t ranges, int64_t hint) {
+  if (hp != 1 || pl.mfma || pl.kv8 || p.head_dim != 128 || pl.heads != 4 || pl.waves > 2 ||
+      p.opt.waves_per_group || p.opt.waves_per_cu || ranges <= 0)
+    return false;
+  const int64_t range = (p.num_indices + ranges - 1) / ranges;
+  const bool aligned = hint > 0 && range > 0 && (__int128)hint * p.batch == p.num_indices &&
+                       (hint % range == 0 || range % hint == 0);
+  const int64_t segments = aligned ? std::max<int64_t>(ranges, p.batch) : ranges + p.batch;
+  return p.num_indices >= kLongSegmentPages * segments;
+}
+
 // Whether a caller's explicit split over 256-byte rows runs 4 wavefronts per workgroup
 // (kShortSplitPages): its workgroups are fewer than the CUs; as many as the CUs, streaming
 // short runs of pages (the mean sequence's pages per split); or up to twice as many, so
@@ -375,6 +391,7 @@ int run(Problem p, bool do_merge, void* stream) {
   int waves_per_pair = 0;   // balanced: workgroups per head chunk
   int seg_cost = 0;         // balanced: pages charged per change of sequence
   int hp = 1;               // balanced: kv heads per workgroup
+  bool longs = false;       // balanced: the build for long segments
   if (pl.balanced && p.opt.window > 0) {
     // a sliding window bounds every sequence's pages: explicit splits of the window's
     // pages, as many as fill the device and fit the workspace
@@ -419,6 +436,7 @@ int run(Problem p, bool do_merge, void* stream) {
       }
       pl.grid = balanced_groups(p, pl, cus, hp);
       waves_per_pair = (int)(pl.grid / (pl.pairs_per_seq / hp));
+      longs = long_segments(p, pl, hp, waves_per_pair, hint);
       // a ragged batch (plan hint: the longest sequence well above the mean): charge each
       // change of sequence in the range split, so that ranges crossing more sequences get
       // fewer pages (a kernel build of its own)
@@ -500,6 +518,7 @@ int run(Problem p, bool do_merge, void* stream) {
   L.kv8 = pl.kv8;
   L.hp = hp;
   L.cost = a.seg_cost > 0;
+  L.longs = longs;
   L.grid = (int)pl.grid;
   if (pl.balanced && pl.chunks > 1) {
     // the chunks of a (range, kv-head group) unit sit kXcds workgroup ids apart: whole

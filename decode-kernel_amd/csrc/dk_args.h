@@ -106,6 +106,17 @@ constexpr int kShortSplitPages = 32;
 #define DK_SEGMENT_COST_PER_WAVE 5
 #endif
 constexpr int kSegmentCostPerWave = DK_SEGMENT_COST_PER_WAVE;
+// Balanced schedule whose mean segment (a run of one sequence's pages inside one range) holds
+// at least this many pages, over 16-bit rows at D = 128 with 3 or 4 q heads per kv head: the
+// build with a page ring without peeled last pages (dk_pass1_balanced, LONG). 32/8/128, us,
+// before vs ring: B=1 ctx 131072 bf16 88.1 vs 84.5, B=4 ctx 32768 bf16 88.0 vs 84.2, B=3 ctx
+// 100000 192.2 vs 183.8, B=16 ctx 4096 (64 pages, ranges on sequence starts) 47.8 vs 45.6, B=1
+// ctx 32768 (64) 28.5 vs 27.4, B=16 ctx 2048 (64) 27.0 vs 26.4, ragged B=128 ctx U[128, 8192]
+// (206) 321.3 vs 312.0, B=100 ctx U[1000, 3000] (95) 143.5 vs 138.3, 16/4 B=32 ctx U[1000,
+// 9000] 60.5 vs 59.0; shorter segments lose: B=5 ctx 6000 (51) 27.6 vs 27.6, B=16 ctx U[300,
+// 4000] (45) 27.6 vs 28.4, B=64 ctx U[100, 2000] (43) 55.3 vs 58.0; and so do 1 or 2 q heads
+// per kv head: 8/8 B=16 ctx U[3000, 9000] 74.4 vs 74.9, 16/8 B=64 270.0 vs 270.7.
+constexpr int64_t kLongSegmentPages = 64;
 // Balanced schedule over narrow rows: 4 neighbouring kv heads per workgroup, 2 wavefronts
 // each, one such workgroup per CU (64- and 128-byte row segments 512 B or 1 KB apart
 // stream far better when the segments of neighbouring heads are fetched together). B=32

@@ -1153,6 +1153,23 @@ __device__ __forceinline__ void stream_ring(W& wv, int n, PageFn page, ValidFn v
   }
 }
 
+// stream_ring at two pages ahead with page 0 already loading in ka / va (the balanced kernel's
+// LONG build): no peeled last pages, a round of three pages per trip.
+template <bool CAP, class W, class PageFn, class ValidFn>
+__device__ __forceinline__ void stream_ring3(W& wv, u32 (&ka)[W::KB], u32 (&va)[W::VB], int n,
+                                             PageFn page, ValidFn valid) {
+  u32 kb[W::KB], vb[W::VB], kc[W::KB], vc[W::VB];
+  wv.load_page(kb, vb, page(min(1, n - 1)), 1 < n);
+  for (int k = 0; k < n; k += 3) {
+    wv.load_page(kc, vc, page(min(k + 2, n - 1)), k + 2 < n);
+    wv.template consume<CAP>(ka, va, valid(k));
+    wv.load_page(ka, va, page(min(k + 3, n - 1)), k + 3 < n);
+    if (k + 1 < n) wv.template consume<CAP>(kb, vb, valid(k + 1));
+    wv.load_page(kb, vb, page(min(k + 4, n - 1)), k + 4 < n);
+    if (k + 2 < n) wv.template consume<CAP>(kc, vc, valid(k + 2));
+  }
+}
+
 // Pages straight into LDS: a ring of DEPTH + 1 page slots per wavefront (`ring`,
 // DEPTH + 1 slots of W::LDS_PAGE bytes); while page k is read and computed, the loads of
 // the next DEPTH pages are in flight without holding registers. hipcc does not order the
@@ -1377,7 +1394,7 @@ constexpr bool first_page_by_caller() {
 // into ka / va; the balanced kernel issues that load before it has found the sequence of
 // its first segment, and before the previous segment's combine for the others
 // (first_page_by_caller kernels only).
-template <int D, bool KV8, bool CAP, bool BAL = false, class WV, class PageFn,
+template <int D, bool KV8, bool CAP, bool BAL = false, bool LONG = false, class WV, class PageFn,
           class ValidFn>
 __device__ __forceinline__ void stream_loaded(WV& wv, int NW, int w, int n, PageFn page,
                                               ValidFn valid, u32 (&ka)[WV::KB],
@@ -1386,8 +1403,10 @@ __device__ __forceinline__ void stream_loaded(WV& wv, int NW, int w, int n, Page
   if (nk > 0) {
     auto pk = [&](int k) { return page(w + NW * k); };
     auto vk = [&](int k) { return valid(w + NW * k); };
-    stream_pages<prefetch_depth<D, KV8, BAL, WV::HEADS, WV::MF>(), CAP, false>(wv, ka, va, nk,
-                                                                               pk, vk);
+    constexpr int depth = prefetch_depth<D, KV8, BAL, WV::HEADS, WV::MF>();
+    static_assert(!LONG || depth == 2, "the long build keeps two pages in flight");
+    if constexpr (LONG) stream_ring3<CAP>(wv, ka, va, nk, pk, vk);
+    else stream_pages<depth, CAP, false>(wv, ka, va, nk, pk, vk);
   }
 }
 
@@ -1523,8 +1542,12 @@ __device__ __forceinline__ int cost_boundary(const Pass1Args& a, int base, int P
 // contiguous and ordered) for the merge kernel.
 // COST: the build whose range split charges sequence starts (a.seg_cost, ragged batches);
 // the other one splits equal pages and carries none of that code.
-template <class T, int D, int G, int NW, bool MFMA, bool KV8, int HP, bool COST = false>
-__global__ __launch_bounds__(NW * HP * 64, (min_waves_per_simd<D, G, KV8>())) void dk_pass1_balanced(Pass1Args a) {
+// LONG: the build for ranges whose segments are long (long_segments in dk_api.hip): the pages
+// stream through stream_ring3 at up to 512 registers (its grid keeps one wavefront per SIMD
+// at most; at 256 the ring's loads are scheduled apart and it loses, 84.8 -> 90.8 us).
+template <class T, int D, int G, int NW, bool MFMA, bool KV8, int HP, bool COST = false,
+          bool LONG = false>
+__global__ __launch_bounds__(NW * HP * 64, (LONG ? 1 : min_waves_per_simd<D, G, KV8>())) void dk_pass1_balanced(Pass1Args a) {
   using WV = Wave<T, D, G, MFMA, KV8>;
   __shared__ CombineSmem<G, D, (NW > 1 ? NW : 1)> smh[HP];
   __shared__ __attribute__((aligned(16))) uint8_t kst[WV::STAGE ? HP * NW * WV::STAGE_BYTES : 16];
@@ -1637,9 +1660,9 @@ __global__ __launch_bounds__(NW * HP * 64, (min_waves_per_simd<D, G, KV8>())) vo
     if constexpr (PRE) {
       // ka / va hold (or are loading) this segment's page w, the range's unit u + w
       if (a.cap_out != 0.f)
-        stream_loaded<D, KV8, true, true>(wv, NW, w, n, page, valid, ka, va);
+        stream_loaded<D, KV8, true, true, LONG>(wv, NW, w, n, page, valid, ka, va);
       else
-        stream_loaded<D, KV8, false, true>(wv, NW, w, n, page, valid, ka, va);
+        stream_loaded<D, KV8, false, true, LONG>(wv, NW, w, n, page, valid, ka, va);
     } else {
       if (a.cap_out != 0.f)
         stream_interleaved<D, KV8, true, LDSP, false, true>(wv, NW, w, n, page, valid, wring);

@@ -881,3 +881,36 @@ def test_plan_schedule_names_the_window_split_that_runs(batch, window):
     explicit = decode_attention(q, kv, indptr, ids, last, split_kv=s, window=window)
     torch.cuda.synchronize()
     assert torch.equal(auto, explicit)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hq,hkv", [(32, 8), (24, 8), (4, 1)])
+@pytest.mark.parametrize("lens,hinted", [
+    ([65536], True), ([65521], False), ([16384] * 4, True),           # ranges on sequence starts
+    ([40000, 1, 0, 17, 49, 20000, 100, 160], True),                   # short and empty ones between
+    ([30011, 29999, 15], False)])
+def test_balanced_long_segments(dtype, hq, hkv, lens, hinted):
+    # the page ring of the long-segment build (mean segment of at least 64 pages): remainders of
+    # its rounds of three pages, soft-capping, with and without the plan hint, against the one
+    # pass over the same pages and the oracle on the shortest sequences
+    print(f"[case] long segments {dtype} {hq}/{hkv} {lens} hint={hinted}", flush=True)
+    if hkv == 1:
+        lens = [8 * n for n in lens]         # 256 ranges of the one kv head
+    q, kv, indptr, ids, last, _ = layout.synthesize_paged(
+        len(lens), lens, hq, hkv, 128, dtype=dtype, device=DEV, page_table="permuted", seed=4)
+    hint = attention.plan_hint(indptr.cpu()) if hinted else 0
+    rows = [b for b, n in enumerate(lens) if n <= 200]
+    want = _oracle(q, kv, indptr, ids, last, batch_subset=rows) if rows else None
+    for cap in (None, 15.0):
+        out = decode_attention(q, kv, indptr, ids, last, 0, max_pages_per_seq=hint, schedule=1,
+                               logit_cap=cap)
+        one = decode_attention(q, kv, indptr, ids, last, 1, logit_cap=cap)
+        torch.cuda.synchronize()
+        # one rounding of the output each, fp32 sums in another order
+        ulp = 2.0 ** (-10 if dtype == torch.float16 else -7)
+        diff = (out.float() - one.float()).abs()
+        assert bool((diff <= ulp * one.float().abs() + 1e-5).all()), float(diff.max())
+        if rows and cap is None:
+            _check(out, want, rows, label="long segments")
+    assert torch.equal(out, decode_attention(q, kv, indptr, ids, last, 0, max_pages_per_seq=hint,
+                                             schedule=1, logit_cap=15.0))
