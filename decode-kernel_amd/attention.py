@@ -299,6 +299,25 @@ class _LibraryScratch:
 
 
 _SCRATCH = _LibraryScratch()
+_NATIVE = None           # _dk_native.decode once bound to the loaded library
+
+
+def _bind_native():
+    """_dk_native.decode (csrc/dk_native.cpp), bound to the loaded library and to torch's
+    stream state. It runs decode_attention's plain calls; for the others it returns None."""
+    global _NATIVE
+    import _dk_native
+    lib = dk_lib.load()
+    address = lambda f: ctypes.cast(f, ctypes.c_void_p).value  # noqa: E731
+    _dk_native.bind(address(lib.dk_decode_attention_ex), address(lib.dk_decode_attention_kv),
+                    address(lib.dk_workspace_bytes), torch.cuda.current_device,
+                    torch._C._cuda_getCurrentRawStream, torch.cuda.is_current_stream_capturing,
+                    lambda index, stream, need: _SCRATCH.get(torch.device("cuda", index), stream,
+                                                             need))
+    _NATIVE = _dk_native.decode
+    return _NATIVE
+
+
 _PLANS: dict = {}
 _PLANS_MAX = 512
 
@@ -454,9 +473,11 @@ def decode_attention(
                            device; head h's softmax gets one more term e^{sinks[h]} that
                            takes weight and carries no value; None = off
 
-    The argument checks run once per call signature (shapes, strides, dtypes, devices and
-    options); later calls with the same signature reuse the validated plan, so a model's
-    layers pay only for the pointers and the library call.
+    Plain calls (16-token pages, contiguous tables, the current device, no graph capture) are
+    checked and launched by _dk_native, at about the cost of their launches. For the others the
+    argument checks run once per call signature (shapes, strides, dtypes, devices and options);
+    later calls with the same signature reuse the validated plan, so a model's layers pay only
+    for the pointers and the library call.
 
     Pages of a multiple of 16 tokens (32, 64, ...; FlashInfer allows any page size, the
     reference only 16) are read in place as 16-token sub-pages: the page table is
@@ -467,6 +488,15 @@ def decode_attention(
     Returns:
         (batch, num_q_heads, head_dim) tensor, same dtype as q.
     """
+    if isinstance(q, torch.Tensor) and q.is_cuda:
+        got = (_NATIVE or _bind_native())(
+            q, kv_data, kv_indptr, kv_indices, kv_last_page_len, split_kv, out, workspace,
+            qk_path, waves_per_group, waves_per_cu, schedule, max_pages_per_seq, sm_scale,
+            k_scale, v_scale, logit_cap, window, sinks)
+        if isinstance(got, int):
+            dk_lib.check(got, "decode_attention")
+        elif got is not None:
+            return got
     ps = _page_size_of(kv_data)
     if ps is not None and ps != PAGE_SIZE and ps > 0 and ps % PAGE_SIZE == 0:
         return _decode_over_sub_pages(

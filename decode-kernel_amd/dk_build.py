@@ -18,6 +18,7 @@ CSRC = HERE / "csrc"
 INCLUDE = HERE.parent / "include"
 LIB_NAME = "libdk_decode.so"
 LIB_PATH = HERE / LIB_NAME
+NATIVE_PATH = HERE / "_dk_native.so"
 BUILD_DIR = HERE / "_build"
 ARCH = "gfx950"
 
@@ -107,6 +108,22 @@ def _run_all(cmds: list[list[str]]) -> str:
     return "\n".join(raw)
 
 
+def native_command() -> list[str]:
+    """The compile of csrc/dk_native.cpp (_dk_native, the call path read through ATen) with
+    this interpreter's and torch's headers."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    lib = Path(torch.__file__).resolve().parent / "lib"
+    return ["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-Wall",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f"-I{sysconfig.get_paths()['include']}", *(f"-I{p}" for p in include_paths()),
+            f"-I{INCLUDE}", str(CSRC / "dk_native.cpp"), "-o", str(NATIVE_PATH) + ".tmp",
+            f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
+
+
 def build(verbose: bool = False, defines: tuple = (), out: Path = LIB_PATH,
           build_dir: Path = BUILD_DIR) -> Path:
     """Compile csrc/ into libdk_decode.so (always rebuilds). Returns the library path.
@@ -131,6 +148,8 @@ def build(verbose: bool = False, defines: tuple = (), out: Path = LIB_PATH,
             objs.append(obj)
             cmds.append([hipcc, *HIP_FLAGS, *dflags, f"-DDK_HEAD_DIM={d}", RESOURCE_FLAG,
                          f"-I{INCLUDE}", "-c", str(CSRC / src), "-o", str(obj)])
+    if out == LIB_PATH:
+        cmds.append(native_command())
     res = kernel_resources(_run_all(cmds))
     (build_dir / "kernel_resources.txt").write_text("".join(
         f"{k} VGPRs={v.get('VGPRs')} scratch={v.get('ScratchSize')} "
@@ -144,6 +163,8 @@ def build(verbose: bool = False, defines: tuple = (), out: Path = LIB_PATH,
     _run_all([[hipcc, "-shared", "-fPIC", f"--offload-arch={ARCH}", *map(str, objs),
                "-o", str(tmp)]])
     os.replace(tmp, out)
+    if out == LIB_PATH:
+        os.replace(str(NATIVE_PATH) + ".tmp", NATIVE_PATH)
     if verbose:
         print(f"built {out}")
     return out
