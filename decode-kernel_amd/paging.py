@@ -26,6 +26,13 @@ def page_capacity(seq_lens_sum: int, batch: int) -> int:
     return (int(seq_lens_sum) + (PAGE_SIZE - 1) * int(batch)) // PAGE_SIZE
 
 
+def _index_array(t: torch.Tensor, dev) -> torch.Tensor:
+    """t on dev, contiguous, int32 or int64 (which the page-table kernel reads as it is)."""
+    if t.dtype != torch.int64:
+        t = t.to(device=dev, dtype=torch.int32)
+    return t.to(device=dev).contiguous()
+
+
 def build_page_table(req_to_token: torch.Tensor, req_pool_indices: torch.Tensor,
                      seq_lens: torch.Tensor, capacity: Optional[int] = None,
                      seq_lens_sum: Optional[int] = None, out=None):
@@ -64,8 +71,7 @@ def build_page_table(req_to_token: torch.Tensor, req_pool_indices: torch.Tensor,
         if seq_lens_sum is None:
             raise DecodeArgumentError("give capacity or seq_lens_sum (a host integer)")
         capacity = page_capacity(seq_lens_sum, batch)
-    rpi = req_pool_indices.to(device=dev, dtype=torch.int32).contiguous()
-    lens = seq_lens.to(device=dev, dtype=torch.int32).contiguous()
+    rpi, lens = _index_array(req_pool_indices, dev), _index_array(seq_lens, dev)
     if out is None:
         kv_indptr = torch.empty(batch + 1, dtype=torch.int32, device=dev)
         kv_indices = torch.empty(max(int(capacity), 1), dtype=torch.int32, device=dev)
@@ -75,9 +81,10 @@ def build_page_table(req_to_token: torch.Tensor, req_pool_indices: torch.Tensor,
         return kv_indptr[:1], kv_indices[:0], kv_last[:0]
     with torch.cuda.device(dev):
         stream = torch.cuda.current_stream(dev).cuda_stream
-        rc = dk_lib.load().dk_build_page_table(
-            req_to_token.data_ptr(), req_to_token.stride(0), rpi.data_ptr(), lens.data_ptr(),
-            batch, PAGE_SIZE, kv_indptr.data_ptr(), kv_indices.data_ptr(), int(capacity),
+        rc = dk_lib.load().dk_build_page_table_wide(
+            req_to_token.data_ptr(), req_to_token.stride(0), rpi.data_ptr(),
+            rpi.dtype == torch.int64, lens.data_ptr(), lens.dtype == torch.int64, batch,
+            PAGE_SIZE, kv_indptr.data_ptr(), kv_indices.data_ptr(), int(capacity),
             kv_last.data_ptr(), stream)
     dk_lib.check(rc, "build_page_table")
     return kv_indptr[:batch + 1], kv_indices[:int(capacity)], kv_last[:batch]

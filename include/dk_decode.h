@@ -263,6 +263,15 @@ int dk_build_page_table(const int32_t* req_to_token, int64_t req_stride,
                         int32_t* kv_indices, int64_t capacity, int32_t* kv_last_page_len,
                         void* hip_stream);
 
+/* dk_build_page_table with req_pool_indices and seq_lens each int32 (0) or int64 (nonzero
+ * rows_int64 / lens_int64; the values as a cast to int32 gives them), as a framework keeps
+ * them: no cast launches before it. */
+int dk_build_page_table_wide(const int32_t* req_to_token, int64_t req_stride,
+                             const void* req_pool_indices, int32_t rows_int64,
+                             const void* seq_lens, int32_t lens_int64, int32_t batch,
+                             int32_t page_size, int32_t* kv_indptr, int32_t* kv_indices,
+                             int64_t capacity, int32_t* kv_last_page_len, void* hip_stream);
+
 /* The page table of a cache with pages of page_size = 16 * s tokens (FlashInfer allows any
  * page size; the reference checks page_size == 16, src/cuda_/attention_ext.cu:508,551)
  * rewritten over its 16-token sub-pages, so the decode entry points (page_size 16) read

@@ -220,6 +220,37 @@ def test_device_page_table_matches_oracle(lens, server_page):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtypes", [(torch.int32, torch.int64), (torch.int64, torch.int32),
+                                    (torch.int16, torch.int64)])
+@pytest.mark.parametrize("lens", [[4096], [4097, 0, 20000, 5], [131072]])
+def test_page_tables_over_several_workgroups(dtypes, lens):
+    # rows and lengths of either integer type; sequences of one to many workgroups' entries
+    print(f"[case] page table {dtypes} {lens}", flush=True)
+    g = torch.Generator()
+    g.manual_seed(1)
+    r2t = torch.randint(0, 1 << 24, (len(lens) + 2, max(lens)), generator=g, dtype=torch.int32)
+    rows = torch.randperm(len(lens) + 2, generator=g)[:len(lens)]
+    indptr, indices, last = paging.build_page_table(
+        r2t.to(DEV), rows.to(DEV, dtypes[0]), torch.tensor(lens, device=DEV, dtype=torch.int64).to(
+            dtypes[1]), seq_lens_sum=sum(lens))
+    wi, wx, wl = ptab.build_page_table(r2t.numpy(), rows.tolist(), lens)
+    total = int(wi[-1])
+    assert indptr.cpu().tolist() == wi.tolist() and last.cpu().tolist() == wl.tolist()
+    assert indices[:total].cpu().tolist() == wx.tolist()
+    # the same pages as a table of 64-token pages, rewritten over its sub-pages
+    pages = [-(-n // 64) for n in lens]
+    ip = torch.tensor([0] + list(np.cumsum(pages)), dtype=torch.int32)
+    ids = torch.randperm(max(sum(pages), 1), generator=g)[:sum(pages)].to(torch.int32)
+    ll = torch.tensor([n - (p - 1) * 64 if p else 64 for n, p in zip(lens, pages)],
+                      dtype=torch.int32)
+    got = paging.expand_page_table(ip.to(DEV), ids.to(DEV), ll.to(DEV), 64, 8, int(sum(pages)))
+    want = ptab.expand_page_table(ip.numpy(), ids.numpy(), ll.numpy(), 64, 8, int(sum(pages)))
+    n = int(want[0][-1])
+    assert got[0].cpu().tolist() == list(want[0]) and got[1][:n].cpu().tolist() == list(want[1][:n])
+    assert got[2].cpu().tolist() == list(want[2])
+
+
+@pytest.mark.gpu
 def test_device_page_table_empty_requests_and_capacity_clamp():
     fb, _, _, r2t = make_batch([0, 40, 0, 16], layers=1, seed=9)
     rows = fb.req_pool_indices.tolist()
