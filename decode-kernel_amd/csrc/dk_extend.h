@@ -33,6 +33,15 @@ namespace dk {
 
 constexpr int kExtendRows = 128;      // query rows per workgroup
 constexpr int kExtendThreads = 256;
+// A call of fewer workgroups than fill the chip splits each query tile's keys over several, so
+// that about kExtendFill (two per CU) run, with at least kExtendSplitKeys keys each for the
+// longest request; fp32 partials and the decode merge kernel put them together. 32/8/128
+// bf16, us, one workgroup per tile -> split: 16 new of 8,016 tokens 246 -> 21 (split 31), 8
+// requests of 16-64 new of 2,000-4,000 tokens 125 -> 64 (split 5); calls that fill the chip
+// keep one (2048 new of 8192 tokens 489 both).
+constexpr int kExtendFill = 512;
+constexpr int kExtendSplitKeys = 256;
+constexpr int kExtendMaxSplit = 32;
 constexpr int kExtendMaxReqs = 128;   // requests per launch (their sizes are kernel arguments)
 
 struct ExtendReq {
@@ -55,6 +64,8 @@ struct ExtendArgs {
   uint32_t k_s, v_s;                   // bytes: token slot
   int64_t req_stride;                  // elements
   int32_t group, hkv, num_reqs, tiles, window;
+  int32_t split;                       // workgroups per query tile, each a range of its keys
+  float *part_o, *part_m, *part_l;     // split > 1: row (token * q heads + head) * split + s
   uint32_t num_slots;
   float kscale;                        // log2(e) * softmax scale * K dequantisation scale (> 0)
   float cap_in, cap_out;               // soft-cap: x = cap_out * tanh(q.k * cap_in)
@@ -138,8 +149,13 @@ __global__ __launch_bounds__(kExtendThreads, (D <= 128 ? 2 : 1)) void dk_extend(
   const bool active = row0 + 32 * w < rows;
   const int bpos0 = prefix + row0 / G, bpos1 = prefix + min(row0 + kExtendRows - 1, rows - 1) / G;
   const int win = a.window > 0 ? a.window : INT32_MAX;
-  const int kbeg = max(bpos0 - win + 1, 0) / BN;
-  const int kend = bpos1 / BN + 1;
+  int kbeg = max(bpos0 - win + 1, 0) / BN;
+  int kend = bpos1 / BN + 1;
+  if (a.split > 1) {                   // this workgroup's range of key tiles (may be empty)
+    const int per = (kend - kbeg + a.split - 1) / a.split;
+    kbeg += (int)blockIdx.y * per;
+    kend = min(kbeg + per, kend);
+  }
 
   u32x4 qf[QK];
   {
@@ -329,6 +345,25 @@ __global__ __launch_bounds__(kExtendThreads, (D <= 128 ? 2 : 1)) void dk_extend(
   }
 
   lsum = sum_xor32(lsum);
+  if (a.split > 1) {
+    // relative to this range's reference max; dk_merge_split adds the sinks and normalises
+    if (row < rows) {
+      const int64_t r = ((int64_t)(rq.q0 + tok) * (a.hkv * G) + kvh * G + head) * a.split +
+                        blockIdx.y;
+#pragma unroll
+      for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          *reinterpret_cast<f32x4*>(a.part_o + r * D + 32 * b + 8 * x + 4 * h) =
+              f32x4{o[b][4 * x] * a.vscale, o[b][4 * x + 1] * a.vscale, o[b][4 * x + 2] * a.vscale,
+                    o[b][4 * x + 3] * a.vscale};
+      if (h == 0) {
+        a.part_m[r] = mref * kLn2;
+        a.part_l[r] = lsum;
+      }
+    }
+    return;
+  }
   if (a.sinks) lsum += __builtin_amdgcn_exp2f(a.sinks[kvh * G + head] * kLog2e - mref);
   const float inv = lsum == 0.f ? 0.f : a.vscale / lsum;
   if (row < rows) {

@@ -10,11 +10,69 @@
 #include "dk_args.h"
 #include "dk_decode.h"
 #include "dk_extend.h"
+#include "dk_launch.h"
+
+namespace dk {
+namespace {
+
+// Workgroups per query tile (kExtendFill): 1 = the keys are not split.
+int extend_split(int32_t batch, const int32_t* new_lens, const int32_t* all_lens, int32_t hkv,
+                 int32_t group, int32_t window) {
+  int64_t groups = 0, keys = 0;
+  for (int32_t b = 0; b < batch; ++b) {
+    if (new_lens[b] <= 0) continue;
+    groups += ((int64_t)new_lens[b] * group + kExtendRows - 1) / kExtendRows * hkv;
+    // a tile of 128 rows spans up to 128 / group + 1 positions beyond its window
+    const int64_t seen = window > 0 ? (int64_t)window + kExtendRows / group + 1 : INT32_MAX;
+    keys = std::max<int64_t>(keys, std::min<int64_t>(all_lens[b], seen));
+  }
+  if (groups == 0) return 1;
+  const int64_t s = std::min<int64_t>(kExtendFill / groups, keys / kExtendSplitKeys);
+  return (int)std::min<int64_t>(std::max<int64_t>(s, 1), kExtendMaxSplit);
+}
+
+template <class T>
+hipError_t merge(const ExtendArgs& a, int64_t tokens, int d, hipStream_t stream) {
+  MergeArgs m{};
+  m.po = a.part_o;
+  m.pm = a.part_m;
+  m.pl = a.part_l;
+  m.out = a.out;
+  m.o_b = a.o_b;
+  m.o_h = a.o_h;
+  m.batch = (int32_t)tokens;
+  m.hq = a.hkv * a.group;
+  m.split = a.split;
+  m.sinks = a.sinks;
+  return launch_merge<T>(m, d, false, stream);
+}
+
+}  // namespace
+}  // namespace dk
+
+extern "C" size_t dk_extend_workspace_bytes(int32_t batch, const int32_t* new_lens,
+                                            const int32_t* all_lens, int32_t num_q_heads,
+                                            int32_t num_kv_heads, int32_t head_dim,
+                                            int32_t window) {
+  using namespace dk;
+  if (batch <= 0 || !new_lens || !all_lens || num_q_heads <= 0 || num_kv_heads <= 0 ||
+      num_q_heads % num_kv_heads != 0 || head_dim <= 0 || window < 0)
+    return 0;
+  const int s = extend_split(batch, new_lens, all_lens, num_kv_heads, num_q_heads / num_kv_heads,
+                             window);
+  if (s == 1) return 0;
+  int64_t tokens = 0;
+  for (int32_t b = 0; b < batch; ++b) tokens += std::max(new_lens[b], 0);
+  size_t o, m, l, total;
+  partials_layout_rows(tokens * num_q_heads * s, head_dim, &o, &m, &l, &total);
+  return total;
+}
 
 extern "C" int dk_extend_attention(
     const void* q, const void* k_pool, const void* v_pool, const int32_t* req_to_token,
     int64_t req_stride, int64_t num_rows, const int32_t* rows, const int32_t* new_lens,
-    const int32_t* all_lens, void* out, int32_t batch, int64_t num_tokens, int32_t num_q_heads,
+    const int32_t* all_lens, void* out, void* workspace, size_t workspace_bytes, int32_t batch,
+    int64_t num_tokens, int32_t num_q_heads,
     int32_t num_kv_heads, int32_t head_dim, int64_t num_slots, int32_t dtype, int32_t kv_dtype,
     const dk_extend_strides* strides, float score_scale, float v_scale, float logit_cap,
     int32_t window, const float* sinks, void* hip_stream) {
@@ -96,6 +154,20 @@ extern "C" int dk_extend_attention(
   a.cap_in = logit_cap != 0.f ? score_scale / logit_cap : 0.f;
   a.cap_out = kLog2e * logit_cap;
   a.vscale = v_scale;
+  // without a workspace for the partials the keys are not split
+  a.split = extend_split(batch, new_lens, all_lens, num_kv_heads, group, window);
+  if (a.split > 1) {
+    size_t off_o, off_m, off_l, total;
+    partials_layout_rows(first * num_q_heads * a.split, head_dim, &off_o, &off_m, &off_l, &total);
+    if (!workspace || workspace_bytes < total || (uintptr_t)workspace % 256 != 0) {
+      a.split = 1;
+    } else {
+      uint8_t* ws = static_cast<uint8_t*>(workspace);
+      a.part_o = reinterpret_cast<float*>(ws + off_o);
+      a.part_m = reinterpret_cast<float*>(ws + off_m);
+      a.part_l = reinterpret_cast<float*>(ws + off_l);
+    }
+  }
   const bool bf16 = dtype == DK_BF16, kv8 = kes == 1, cap = logit_cap != 0.f;
   const void* fn = head_dim == 64    ? extend_symbol<64>(bf16, kv8, cap)
                    : head_dim == 128 ? extend_symbol<128>(bf16, kv8, cap)
@@ -123,9 +195,15 @@ extern "C" int dk_extend_attention(
     a.tiles = (int32_t)tiles;
     void* args[] = {&a};
     const hipError_t e =
-        hipLaunchKernel(fn, dim3((uint32_t)(tiles * num_kv_heads)), dim3(kExtendThreads), args, 0,
+        hipLaunchKernel(fn, dim3((uint32_t)(tiles * num_kv_heads), a.split), dim3(kExtendThreads), args, 0,
                         static_cast<hipStream_t>(hip_stream));
     if (e != hipSuccess) return set_error((int)e, "extend launch: %s", hipGetErrorString(e));
+  }
+  if (a.split > 1) {
+    const hipStream_t st = static_cast<hipStream_t>(hip_stream);
+    const hipError_t e =
+        bf16 ? merge<BF16>(a, first, head_dim, st) : merge<F16>(a, first, head_dim, st);
+    if (e != hipSuccess) return set_error((int)e, "extend merge launch: %s", hipGetErrorString(e));
   }
   return DK_OK;
 }

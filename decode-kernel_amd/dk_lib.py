@@ -105,9 +105,11 @@ SIGNATURES = {
                                         _I32, _I32, _I32, _I32, _I32, _I32, _I64, _I64, _I32,
                                         ctypes.c_float, ctypes.c_float,
                                         ctypes.POINTER(DkStrides), _P]),
+    "dk_extend_workspace_bytes": (_SZ, [_I32, ctypes.POINTER(_I32), ctypes.POINTER(_I32), _I32,
+                                        _I32, _I32, _I32]),
     "dk_extend_attention": (ctypes.c_int, [_P, _P, _P, _P, _I64, _I64, ctypes.POINTER(_I32),
-                                           ctypes.POINTER(_I32), ctypes.POINTER(_I32), _P, _I32,
-                                           _I64, _I32, _I32, _I32, _I64, _I32, _I32,
+                                           ctypes.POINTER(_I32), ctypes.POINTER(_I32), _P, _P, _SZ,
+                                           _I32, _I64, _I32, _I32, _I32, _I64, _I32, _I32,
                                            ctypes.POINTER(DkExtendStrides), ctypes.c_float,
                                            ctypes.c_float, ctypes.c_float, _I32, _P, _P]),
     "dk_decode_partials": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _SZ, _I32, _I32, _I32, _I32,

@@ -93,12 +93,17 @@ def extend_attention(q, k_pool, v_pool, req_to_token, rows: Sequence[int],
     s = dk_lib.DkExtendStrides(q.stride(0), q.stride(1), k_pool.stride(0), k_pool.stride(1),
                                v_pool.stride(0), v_pool.stride(1), out.stride(0), out.stride(1))
     kv8 = k_pool.dtype == attention.KV_FP8
+    lib = dk_lib.load()
+    hq, hkv, d = q.shape[1], k_pool.shape[1], q.shape[2]
+    news, alls = ints(*new_lens), ints(*all_lens)
+    need = lib.dk_extend_workspace_bytes(n, news, alls, hq, hkv, d, window or 0)
+    ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
     with torch.cuda.device(q.device):
-        rc = dk_lib.load().dk_extend_attention(
+        rc = lib.dk_extend_attention(
             q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(), req_to_token.data_ptr(),
-            req_to_token.stride(0), n_rows, ints(*(r % n_rows for r in rows)), ints(*new_lens),
-            ints(*all_lens), out.data_ptr(), n, q.shape[0], q.shape[1], k_pool.shape[1],
-            q.shape[2], k_pool.shape[0], attention._DTYPE_CODE[q.dtype],
+            req_to_token.stride(0), n_rows, ints(*(r % n_rows for r in rows)), news, alls,
+            out.data_ptr(), None if ws is None else ws.data_ptr(), need, n, q.shape[0], hq, hkv, d,
+            k_pool.shape[0], attention._DTYPE_CODE[q.dtype],
             dk_lib.DK_KV_FP8_E4M3 if kv8 else dk_lib.DK_KV_SAME, ctypes.byref(s),
             scale * k_scale, v_scale, logit_cap or 0.0, window or 0,
             None if sinks is None else sinks.data_ptr(),

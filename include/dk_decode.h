@@ -334,6 +334,11 @@ typedef struct dk_extend_strides {
   int64_t q_b, q_h, k_s, k_h, v_s, v_h, o_b, o_h;
 } dk_extend_strides;
 
+/* Bytes of fp32 scratch that dk_extend_attention can use for these sizes (HOST arrays); 0: none. */
+size_t dk_extend_workspace_bytes(int32_t batch, const int32_t* new_lens, const int32_t* all_lens,
+                                 int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                                 int32_t window);
+
 /* Extend (prefill) attention over a token pool: request b's new_lens[b] new tokens are the
  * last of its all_lens[b] tokens; new token i (position p = all_lens[b] - new_lens[b] + i)
  * attends to positions <= p (with window > 0, to the last `window` of them), whose K and V
@@ -345,12 +350,16 @@ typedef struct dk_extend_strides {
  * logit_cap != 0; the output is scaled by v_scale; sinks as in dk_options. rows, new_lens and
  * all_lens are HOST arrays of `batch` entries, read before the call returns; the rest is
  * device memory, used on hip_stream. req_to_token rows are req_stride entries apart,
- * num_rows of them. The SGLang prefill path (the reference leaves it to other libraries,
+ * num_rows of them. With dk_extend_workspace_bytes of 256-byte aligned workspace, a call of few
+ * new tokens over long contexts splits the keys over more workgroups and merges them (fewer
+ * bytes, or NULL, affect speed only; calls that share one must not overlap in time). The
+ * SGLang prefill path (the reference leaves it to other libraries,
  * integration/sglang_backend.py:94-99). */
 int dk_extend_attention(const void* q, const void* k_pool, const void* v_pool,
                         const int32_t* req_to_token, int64_t req_stride, int64_t num_rows,
                         const int32_t* rows, const int32_t* new_lens, const int32_t* all_lens,
-                        void* out, int32_t batch, int64_t num_tokens, int32_t num_q_heads,
+                        void* out, void* workspace, size_t workspace_bytes, int32_t batch,
+                        int64_t num_tokens, int32_t num_q_heads,
                         int32_t num_kv_heads, int32_t head_dim, int64_t num_slots, int32_t dtype,
                         int32_t kv_dtype, const dk_extend_strides* strides, float score_scale,
                         float v_scale, float logit_cap, int32_t window, const float* sinks,

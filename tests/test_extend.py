@@ -112,6 +112,23 @@ def test_many_requests_and_long_context(monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 64), (torch.bfloat16, 128),
+                                     (torch.bfloat16, 256)])
+@pytest.mark.parametrize("new,pre,win,sinks", [
+    ([1], [4000], None, False), ([16, 3], [3000, 10], None, True), ([40], [600], None, False),
+    ([5, 2], [2000, 1500], 700, False), ([130], [0], None, True), ([9], [511], None, False)])
+def test_keys_split_over_workgroups(monkeypatch, dtype, d, new, pre, win, sinks):
+    # few new tokens over long prefixes: ranges of keys per workgroup, some empty for the shorter
+    # requests, merged; and the same call without the workspace, unsplit
+    print(f"[case] extend split {dtype} d={d} new={new} pre={pre} win={win}", flush=True)
+    fb, layer, pool, qkv = _batch(new, pre, 8, 2, d, dtype, seed=12, win=win)
+    q, k, v = (t.contiguous() for t in qkv.split([8, 2, 2], dim=1))
+    kw = {"sinks": torch.randn(8, device=DEV)} if sinks else {}
+    got, want = _both(monkeypatch, fb, layer, q, k, v, **kw)
+    _close(got, want)
+
+
+@pytest.mark.gpu
 def test_slots_and_rows_count_from_the_end(monkeypatch):
     # negative slots and rows index as PyTorch does; pools as strided views of one buffer
     fb, layer, pool, qkv = _batch([20, 9], [30, 0], 8, 2, 128, torch.float16, seed=8)
@@ -162,6 +179,21 @@ def test_host_tensors_stay_on_pytorch():
                             [9], 0.1, None, 1.0, 1.0, None)
 
 
+def test_split_follows_the_sizes():
+    # bytes of (O, m, l) rows: tokens * heads * split * (d + 2) floats
+    def split(new, alls, hq=32, hkv=8, d=128, win=0):
+        ints = ctypes.c_int32 * len(new)
+        b = dk_lib.load().dk_extend_workspace_bytes(len(new), ints(*new), ints(*alls), hq, hkv, d,
+                                                    win)
+        return b / (4 * sum(new) * hq * (d + 2)) if b else 1
+
+    assert split([2048], [8192]) == 1                     # fills the chip by itself
+    assert split([16], [200]) == 1                        # too few keys
+    assert 31 < split([16], [8192]) < 33 and 15 < split([64], [4096]) < 17
+    assert 1.9 < split([16], [8192], win=512) < 2.1       # bounded by the window
+    assert split([0], [100]) == 1
+
+
 def test_argument_checks():
     # refused before any device call, so without a GPU
     lib = dk_lib.load()
@@ -171,7 +203,7 @@ def test_argument_checks():
         ints = ctypes.c_int32 * len(rows)
         s = dk_lib.DkExtendStrides(hq * d, d, k_s, d, k_s, d, hq * d, d)
         return lib.dk_extend_attention(ptr, ptr, ptr, ptr, stride, num_rows, ints(*rows),
-                                       ints(*new), ints(*alls), ptr, len(rows), tokens, hq, hkv,
+                                       ints(*new), ints(*alls), ptr, None, 0, len(rows), tokens, hq, hkv,
                                        d, 16, dtype, 0, ctypes.byref(s), scale, 1.0, 0.0, window,
                                        None, None)
 
