@@ -14,8 +14,8 @@
 //     the contraction's 16 keys are taken in the order 4h..4h+3, 8+4h..8+4h+3. V^T comes in
 //     that order from the row-major V tile by LDS transpose reads (ds_read_b64_tr_b16).
 //     Each lane's accumulators all belong to its own query row, so rescaling is in-lane.
-//   * p enters as a sum of parts of the element type, 2 in fp16 and 3 in bf16: 22 and 24 bits,
-//     what fp32 weights hold. Scores, softmax, sums and accumulators are fp32.
+//   * p enters as a sum of parts of the element type, 2 in fp16 and 3 in bf16 (ExtendParts).
+//     Scores, softmax, sums and accumulators are fp32.
 // Bound by the matrix cores: in bf16 at D = 128 the four MFMA streams (q.k and the 3 parts of
 // p) run at 1100 TFLOP/s of a large library product's 1267. 32/8/128 bf16, 2048 new of 8192
 // tokens: 437 us (551 TFLOP/s of attention; 371 us in fp16), the PyTorch path 6,200 us; 8
@@ -92,21 +92,36 @@ __device__ __forceinline__ u32x2 lds_read_tr(const uint8_t* p) {
                                        (__attribute__((address_space(3))) i16x4*)p));
 }
 
-// Parts of the element type that a weight is split into. The error of the bf16 output against
-// float64 with 3 parts is that of fp32 weights (1.660468e-3 of the norm at 2048 new of 8192
-// tokens, 32/8/128), 1e-6 of itself more with 2, which would be 12 % faster; fp16 with 2 is
-// below fp32 weights (2.070652e-4 vs 2.070659e-4).
+// Parts of the element type that a weight p = 2^(x - reference) is split into. bf16, 3 parts: 24
+// bits of every weight, as its exponents are fp32's; a row's reference follows its running
+// maximum. The output's error against float64 is that of fp32 weights (1.660468e-3 of the norm
+// at 2048 new of 8192 tokens, 32/8/128), 1e-6 of itself more with 2 parts, which would be 12 %
+// faster.
 template <class T>
 struct ExtendParts {
-  static constexpr int n = 2;
-};
-template <>
-struct ExtendParts<BF16> {
   static constexpr int n = 3;
 };
+// fp16, 2 parts: 22 bits of a weight >= 2^-3, steps of 2^-24 below that. So a row's reference
+// follows its tiles, up and DOWN (a first token may draw most of the attention, and the fp32
+// sums have room): it moves when a tile's largest weight would leave [1, 2^kExtendTop] (fp16
+// ends at 2^16), to where that weight is 2^kExtendMid, or 2^kExtendJump where it lies far above
+// the tiles before it and perhaps above its neighbours too. Error of the weighted sum against
+// float64 in a CPU model of this loop, 8192 keys, one of them with V = 0 and 0 / 14 / 16 / 18
+// nats above the others: 3e-7 / 4e-7 / 3e-7 / 5e-7, of fp32 weights 2e-7 / 3e-7 / 4e-7 / 5e-7,
+// with the running maximum as reference 3e-7 / 9e-5 / 3e-3 / 7e-2; the output's own rounding is
+// 2e-4. Moves are rare but for scores of a wide spread: 2048 new of 8192 tokens, 32/8/128, us,
+// running maximum vs this: scores of 1 nat 374 vs 376, of 3 nats 371 vs 388; D = 64 227 vs 229.
+template <>
+struct ExtendParts<F16> {
+  static constexpr int n = 2;
+};
+constexpr float kExtendTop = 15.5f, kExtendMid = 8.f, kExtendJump = 14.f;
+// The reference never moves further down than leaves the row's sum of weights at 2^kExtendRoom:
+// values of up to 2^16 times that, over any number of keys, stay far from fp32's 2^128.
+constexpr float kExtendRoom = 64.f;
 
 template <class T, int D, bool KV8, bool CAP>
-__global__ __launch_bounds__(kExtendThreads, (D <= 128 ? 2 : 1)) void dk_extend(ExtendArgs a) {
+__global__ __launch_bounds__(kExtendThreads, (D == 64 ? 3 : D == 128 ? 2 : 1)) void dk_extend(ExtendArgs a) {
   constexpr int BN = D <= 128 ? 64 : 32;          // keys per tile
   constexpr int RB = 2 * D;                       // bytes per LDS row
   constexpr int TILE = BN * RB;
@@ -282,8 +297,16 @@ __global__ __launch_bounds__(kExtendThreads, (D <= 128 ? 2 : 1)) void dk_extend(
       for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[n][i]);
     mx = max_xor32(mx);
     if constexpr (!CAP) mx *= a.kscale;
-    if (__builtin_amdgcn_ballot_w64(mx > mref + kSlack)) {
-      const float mn = fmaxf(mref, mx);
+    constexpr bool follow = NP == 2;   // the reference follows the tiles (ExtendParts<F16>)
+    const bool move = follow ? fabsf(mx - (mref + kExtendTop / 2)) > kExtendTop / 2
+                             : mx > mref + kSlack;
+    if (__builtin_amdgcn_ballot_w64(move)) {
+      float mn = fmaxf(mref, mx);
+      if constexpr (follow) {
+        const float to = mx - (mx > mref + kExtendTop + kExtendMid ? kExtendJump : kExtendMid);
+        const float room = __builtin_amdgcn_logf(sum_xor32(lsum)) - kExtendRoom;   // log2
+        mn = mx > kNegInf ? fmaxf(to, mref + room) : mref;   // no key of the tile seen: stays
+      }
       const float al = __builtin_amdgcn_exp2f(mref - mn);
       lsum *= al;
 #pragma unroll
@@ -346,7 +369,7 @@ __global__ __launch_bounds__(kExtendThreads, (D <= 128 ? 2 : 1)) void dk_extend(
 
   lsum = sum_xor32(lsum);
   if (a.split > 1) {
-    // relative to this range's reference max; dk_merge_split adds the sinks and normalises
+    // relative to this range's reference; dk_merge_split adds the sinks and normalises
     if (row < rows) {
       const int64_t r = ((int64_t)(rq.q0 + tok) * (a.hkv * G) + kvh * G + head) * a.split +
                         blockIdx.y;

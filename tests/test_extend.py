@@ -128,6 +128,60 @@ def test_keys_split_over_workgroups(monkeypatch, dtype, d, new, pre, win, sinks)
     _close(got, want)
 
 
+def _direct(q, kp, vp, r2t, row, pre, workspace=True, win=None, sinks=None):
+    """The C ABI's call for one request, with its workspace or without one (keys not split)."""
+    n, hq, d = q.shape
+    hkv, ints = kp.shape[1], ctypes.c_int32 * 1
+    lib = dk_lib.load()
+    new, alls = ints(n), ints(n + pre)
+    out = torch.full_like(q, float("nan"))
+    need = lib.dk_extend_workspace_bytes(1, new, alls, hq, hkv, d, win or 0) if workspace else 0
+    ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
+    s = dk_lib.DkExtendStrides(q.stride(0), d, kp.stride(0), d, vp.stride(0), d, out.stride(0), d)
+    rc = lib.dk_extend_attention(
+        q.data_ptr(), kp.data_ptr(), vp.data_ptr(), r2t.data_ptr(), r2t.stride(0), r2t.shape[0],
+        ints(row), new, alls, out.data_ptr(), None if ws is None else ws.data_ptr(), need, 1, n,
+        hq, hkv, d, kp.shape[0], 0 if q.dtype == torch.float16 else 1, dk_lib.DK_KV_SAME,
+        ctypes.byref(s), d ** -0.5, 1.0, 0.0, win or 0,
+        None if sinks is None else sinks.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    dk_lib.check(rc, "dk_extend_attention")
+    return out, need
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("new,pre,at,nats", [(40, 90, 0, 14), (40, 90, 70, 18), (130, 4000, 0, 16),
+                                             (130, 4000, 0, 18), (33, 8000, 4100, 18),
+                                             (33, 8000, 0, 24), (33, 8000, 0, 60)])
+def test_a_key_that_draws_most_of_the_weight(dtype, d, new, pre, at, nats):
+    # a key `nats` above the others whose V is zero: the output is what the small weights sum
+    # to. Against float64 the error may be that of rounding the output once, 1 % more at most:
+    # beside a rounding of 2e-4 that is an error of the weights below 3e-5 (at 24 nats the
+    # outputs are fp16 subnormals, whose rounding is larger; at 60 they are zero)
+    print(f"[case] extend peaked {dtype} d={d} new={new} pre={pre} at={at} nats={nats}", flush=True)
+    hq, hkv, n = 8, 2, new + pre
+    g = torch.Generator(device=DEV).manual_seed(21)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)  # noqa: E731
+    q, kp, vp = rnd(new, hq, d), rnd(n + 16, hkv, d), 64 + 4 * rnd(n + 16, hkv, d)
+    r2t = torch.randperm(n + 16, generator=g, device=DEV)[:n].int()[None]
+    q[..., 0], kp[..., 0] = 8.0, 0.0
+    kp[r2t[0, at].long(), :, 0] = nats * d ** 0.5 / 8.0
+    vp[r2t[0, at].long()] = 0.0
+    q, kp, vp = q.to(dtype), kp.to(dtype), vp.to(dtype)
+    kk, vv = kp[r2t[0].long()].double(), vp[r2t[0].long()].double()
+    mask = torch.arange(n, device=DEV)[None] > torch.arange(pre, n, device=DEV)[:, None]
+    want = torch.stack([
+        torch.softmax((q[:, i].double() @ kk[:, i // 4].T.contiguous() * d ** -0.5).masked_fill(
+            mask, -math.inf), -1) @ vv[:, i // 4] for i in range(hq)], 1)
+    rounding = float((want.to(dtype).double() - want).norm())
+    for workspace in (True, False):
+        got, need = _direct(q, kp, vp, r2t, 0, pre, workspace)
+        assert (need > 0) == (workspace and n >= 512)          # both ways of the kernel
+        err = float((got.double() - want).norm())
+        assert err <= 1.01 * rounding, (workspace, err / float(want.norm()), rounding / float(want.norm()))
+
+
 @pytest.mark.gpu
 def test_slots_and_rows_count_from_the_end(monkeypatch):
     # negative slots and rows index as PyTorch does; pools as strided views of one buffer
