@@ -7,6 +7,7 @@ adapter on an SGLang-shaped token pool against the oracle, the page table agains
 oracle/page_table.py (bit-exact), split caches and custom scales against the oracle.
 """
 import math
+import re
 
 import numpy as np
 import pytest
@@ -523,6 +524,73 @@ def test_hip_graph_capture_and_replay():
         torch.cuda.synchronize()
         assert torch.equal(big, big_keep), "a graph replay wrote into an eager tensor"
         del big_fb, big_layers, big_pool, big, big_keep
+
+
+def _captured_pass1(graph, path):
+    """Names of the pass-1 kernels in a captured graph."""
+    graph.debug_dump(str(path))
+    return re.findall(r"dk_pass1_[a-z]+I\w+", path.read_text())
+
+
+@pytest.mark.gpu
+def test_captured_step_of_short_sequences_in_a_large_table(tmp_path):
+    # the persistent table has room for 8 requests of 8192 tokens (4104 entries, over 100 per
+    # range and request); the captured call must not take that for long sequences: its kernel
+    # is the one of an eager step without a hint over the batch's own table
+    from types import SimpleNamespace
+    full = [40, 17, 300, 5]
+    fb, layers, pool, r2t = make_batch(full, layers=1, seed=9)
+    rows = fb.req_pool_indices
+    mr = SimpleNamespace(req_to_token_pool=fb.req_to_token_pool, device=DEV,
+                         model_config=SimpleNamespace(context_len=8192))
+    backend = sglang_backend.SplitKVHipBackend(mr)
+    backend.init_cuda_graph_state(max_bs=8)
+    q = torch.randn(4, 32 * 128, generator=torch.Generator(device=DEV).manual_seed(3),
+                    device=DEV).half()
+    backend.init_forward_metadata_capture_cuda_graph(4, 4, rows, fb.seq_lens)
+    backend.forward_decode(q, None, None, layers[0], fb)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    graph.enable_debug_mode()
+    with torch.cuda.graph(graph):
+        out = backend.forward_decode(q, None, None, layers[0], fb)
+    graph.instantiate()
+    for back in (0, 4, 0):
+        lens = [n - back for n in full]
+        fb.seq_lens.copy_(torch.tensor(lens, device=DEV))
+        print(f"[case] graph over a large table lens={lens}", flush=True)
+        backend.init_forward_metadata_replay_cuda_graph(4, rows, fb.seq_lens)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = _want(q.view(-1, 32, 128), pool, 0, r2t.numpy(), rows.tolist(), lens)
+        mx, mean = err_stats(out.view(-1, 32, 128), want)
+        assert mx <= 1e-2 and mean <= 1e-3, (lens, mx, mean)
+    names = _captured_pass1(graph, tmp_path / "step.dot")
+    assert len(names) == 1 and "balanced" in names[0] and names[0].endswith("Lb0EEEvNS_9Pass1ArgsE")
+
+
+@pytest.mark.gpu
+def test_captured_long_sequence_with_its_hint_takes_the_long_build(tmp_path):
+    # ... while a caller that plans a captured call (max_pages_per_seq) keeps that build
+    q, kv, indptr, ids, last, _ = layout.synthesize(1, 16 * 4096, 32, 8, 128, device=DEV, seed=1)
+    names = {}
+    for hint in (0, 4096):
+        want = attention.decode_attention(q, kv, indptr, ids, last, None, max_pages_per_seq=hint)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        graph.enable_debug_mode()
+        with torch.cuda.graph(graph):
+            out = attention.decode_attention(q, kv, indptr, ids, last, None,
+                                             max_pages_per_seq=hint)
+        graph.instantiate()
+        for _ in range(2):
+            graph.replay()
+            torch.cuda.synchronize()
+            # the two builds take a range's pages in the same order: equal to rounding
+            assert float((out.float() - want.float()).abs().max()) <= 1e-3
+        (names[hint],) = _captured_pass1(graph, tmp_path / f"{hint}.dot")
+    assert names[0].endswith("Lb0EEEvNS_9Pass1ArgsE") and names[4096].endswith(
+        "Lb1EEEvNS_9Pass1ArgsE"), names
 
 
 @pytest.mark.gpu
