@@ -22,6 +22,9 @@ from __future__ import annotations
 
 import ctypes
 import math
+import re
+import sys
+import warnings
 from types import SimpleNamespace
 from typing import Optional
 
@@ -304,10 +307,24 @@ _NATIVE = None           # _dk_native.decode once bound to the loaded library
 
 def _bind_native():
     """_dk_native.decode (csrc/dk_native.cpp), bound to the loaded library and to torch's
-    stream state. It runs decode_attention's plain calls; for the others it returns None."""
+    stream state. It runs decode_attention's plain calls; for the others it returns None.
+    Where the extension is missing or was compiled against another library interface, torch
+    or Python, every call is left to the Python path (the same kernels), with one warning."""
     global _NATIVE
-    import _dk_native
     lib = dk_lib.load()
+    runs = (lib.dk_abi_version(), ctypes.sizeof(dk_lib.DkOptions), ctypes.sizeof(dk_lib.DkStrides),
+            re.match(r"[\d.]*\d", torch.__version__).group(), *sys.version_info[:2])
+    try:
+        import _dk_native
+        built = getattr(_dk_native, "BUILT_FOR", None)
+        if built != runs:
+            raise ImportError(f"built for {built}, running {runs}")
+    except ImportError as exc:
+        _NATIVE = lambda *args: None  # noqa: E731
+        warnings.warn(f"_dk_native is not usable ({exc}): decode_attention's calls cost about 5 us "
+                      "more on the host; build it with `python __graft_entry__.py build`",
+                      RuntimeWarning, stacklevel=3)
+        return _NATIVE
     address = lambda f: ctypes.cast(f, ctypes.c_void_p).value  # noqa: E731
     _dk_native.bind(address(lib.dk_decode_attention_ex), address(lib.dk_decode_attention_kv),
                     address(lib.dk_workspace_bytes), torch.cuda.current_device,

@@ -12,6 +12,7 @@
 #include <ATen/ATen.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <cmath>
 #include <cstdint>
@@ -266,4 +267,18 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_dk_native", nullptr, -1, kMethod
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__dk_native() { return PyModule_Create(&kModule); }
+// BUILT_FOR: what this file was compiled against (the C ABI's version and struct sizes, torch,
+// Python); attention.py binds it only where all of it is what runs.
+PyMODINIT_FUNC PyInit__dk_native() {
+  PyObject* m = PyModule_Create(&kModule);
+  if (!m) return nullptr;
+  PyObject* built = Py_BuildValue("(iiisii)", DK_ABI_VERSION, (int)sizeof(dk_options),
+                                  (int)sizeof(dk_strides), TORCH_VERSION, PY_MAJOR_VERSION,
+                                  PY_MINOR_VERSION);
+  if (!built || PyModule_AddObject(m, "BUILT_FOR", built) != 0) {
+    Py_XDECREF(built);
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

@@ -1,5 +1,9 @@
 """decode_attention's native call path (_dk_native) against its Python path: the same bits where
 it takes a call, and the Python path's result or error for every call that it leaves."""
+import sys
+import warnings
+from types import SimpleNamespace
+
 import pytest
 import torch
 
@@ -121,3 +125,47 @@ def test_left_to_python_without_a_gpu():
     assert _dk_native.decode(*(None,) * 19) is None
     with pytest.raises(TypeError):
         _dk_native.decode(q)
+
+
+def _refuse_bind(*args):
+    raise AssertionError("bound an extension that does not fit")
+
+
+def _other(at, value):
+    built = list(_dk_native.BUILT_FOR)
+    built[at] = value
+    return SimpleNamespace(BUILT_FOR=tuple(built), bind=_refuse_bind, decode=_refuse_bind)
+
+
+# missing, too old to say what it fits, another interface version, struct size, torch, Python
+UNUSABLE = [None, SimpleNamespace(bind=_refuse_bind), _other(0, 2), _other(1, 48), _other(2, 56),
+            _other(3, "2.9.1"), _other(5, 9)]
+
+
+@pytest.mark.parametrize("module", UNUSABLE)
+def test_an_extension_that_does_not_fit_leaves_every_call_to_python(monkeypatch, module):
+    monkeypatch.setattr(attention, "_NATIVE", None)
+    monkeypatch.setitem(sys.modules, "_dk_native", module)
+    with pytest.warns(RuntimeWarning, match="__graft_entry__.py build"):
+        bound = attention._bind_native()
+    assert attention._NATIVE is bound and bound(*range(19)) is None
+
+
+def test_the_built_extension_fits(monkeypatch):
+    monkeypatch.setattr(attention, "_NATIVE", None)
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert attention._bind_native() is _dk_native.decode
+
+
+@pytest.mark.gpu
+def test_calls_run_without_the_extension(monkeypatch):
+    args = _inputs()
+    want = decode_attention(*args, 4)
+    monkeypatch.setattr(attention, "_NATIVE", None)
+    monkeypatch.setitem(sys.modules, "_dk_native", None)
+    with pytest.warns(RuntimeWarning):
+        got = decode_attention(*args, 4)
+    with warnings.catch_warnings():       # said once
+        warnings.simplefilter("error")
+        assert torch.equal(decode_attention(*args, 4), want) and torch.equal(got, want)
