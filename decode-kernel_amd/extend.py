@@ -29,7 +29,8 @@ def _aligned(t: torch.Tensor) -> bool:
 def _plain(*tensors: torch.Tensor) -> bool:
     """Ordinary tensors outside tracing, transforms and gradients: what a call that hands
     out raw pointers may take."""
-    if torch._C._len_torch_dispatch_stack() > 0 or torch.autograd.forward_ad._current_level >= 0:
+    if torch._C._len_torch_dispatch_stack() > 0 or torch._C._get_tracing_state() is not None or \
+            torch.autograd.forward_ad._current_level >= 0:
         return False
     grad = torch.is_grad_enabled()
     return all(type(t) is torch.Tensor and not (grad and t.requires_grad) and

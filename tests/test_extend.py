@@ -223,6 +223,26 @@ def test_calls_left_to_pytorch(monkeypatch):
     _close(backend.forward_extend(q, k, v, layer, fb), want)
 
 
+@pytest.mark.gpu
+def test_a_traced_call_records_its_attention():
+    # a call under torch.jit.trace stays on PyTorch, so that the trace computes new inputs
+    fb, layer, pool, qkv = _batch([5, 2], [40, 0], 4, 2, 64, torch.float16, seed=14)
+    pool.get_key_buffer, pool.get_value_buffer = pool.k_buffer.__getitem__, pool.v_buffer.__getitem__
+    backend = sglang_backend.SplitKVHipBackend()
+    call = lambda q: backend.forward_extend(q, None, None, layer, fb)  # noqa: E731
+    q = qkv[:, :4].contiguous()
+    traced = torch.jit.trace(call, (q,), check_trace=False)
+    other = q.flip(0).contiguous()
+    _close(traced(other), call(other))
+
+
+def test_what_passes_tensors_through_a_trace_is_not_plain():
+    t = torch.zeros(2, 4, 64, dtype=torch.float16)
+    seen = []
+    torch.jit.trace(lambda x: (seen.append(extend._plain(x)), x + 1)[1], (t,), check_trace=False)
+    assert seen == [False] and extend._plain(t)
+
+
 def test_host_tensors_stay_on_pytorch():
     fb, layer, pool, qkv = _batch([5, 2], [4, 0], 4, 2, 64, torch.float16, seed=11, device="cpu")
     q, k, v = (t.contiguous() for t in qkv.split([4, 2, 2], dim=1))
