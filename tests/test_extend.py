@@ -111,6 +111,30 @@ def test_many_requests_and_long_context(monkeypatch):
     _close(*_both(monkeypatch, fb, layer, q, k, v))
 
 
+def _direct(q, kp, vp, r2t, rows, new, pre, workspace=True, win=None, sinks=None):
+    """The C ABI's call with its workspace, without one (False), or with one that it cannot use
+    ("short", "unaligned"); returns (out, the workspace's bytes)."""
+    t, hq, d = q.shape
+    hkv, n = kp.shape[1], len(new)
+    ints = ctypes.c_int32 * n
+    lib = dk_lib.load()
+    news, alls = ints(*new), ints(*(a + b for a, b in zip(new, pre)))
+    out = torch.full_like(q, float("nan"))
+    need = lib.dk_extend_workspace_bytes(n, news, alls, hq, hkv, d, win or 0)
+    ws = torch.empty(need + 256, dtype=torch.uint8, device=q.device)
+    at, size = {True: (ws.data_ptr(), need), False: (None, 0), "short": (ws.data_ptr(), need - 1),
+                "unaligned": (ws.data_ptr() + 16, need)}[workspace]
+    s = dk_lib.DkExtendStrides(q.stride(0), d, kp.stride(0), d, vp.stride(0), d, out.stride(0), d)
+    rc = lib.dk_extend_attention(
+        q.data_ptr(), kp.data_ptr(), vp.data_ptr(), r2t.data_ptr(), r2t.stride(0), r2t.shape[0],
+        ints(*rows), news, alls, out.data_ptr(), at, size, n, t, hq, hkv, d, kp.shape[0],
+        0 if q.dtype == torch.float16 else 1, dk_lib.DK_KV_SAME, ctypes.byref(s), d ** -0.5, 1.0,
+        0.0, win or 0, None if sinks is None else sinks.data_ptr(),
+        torch.cuda.current_stream().cuda_stream)
+    dk_lib.check(rc, "dk_extend_attention")
+    return out, need
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype,d", [(torch.float16, 64), (torch.bfloat16, 128),
                                      (torch.bfloat16, 256)])
@@ -119,33 +143,23 @@ def test_many_requests_and_long_context(monkeypatch):
     ([5, 2], [2000, 1500], 700, False), ([130], [0], None, True), ([9], [511], None, False)])
 def test_keys_split_over_workgroups(monkeypatch, dtype, d, new, pre, win, sinks):
     # few new tokens over long prefixes: ranges of keys per workgroup, some empty for the shorter
-    # requests, merged; and the same call without the workspace, unsplit
+    # requests, merged; and the same call without a workspace that it can use, unsplit
     print(f"[case] extend split {dtype} d={d} new={new} pre={pre} win={win}", flush=True)
     fb, layer, pool, qkv = _batch(new, pre, 8, 2, d, dtype, seed=12, win=win)
     q, k, v = (t.contiguous() for t in qkv.split([8, 2, 2], dim=1))
     kw = {"sinks": torch.randn(8, device=DEV)} if sinks else {}
     got, want = _both(monkeypatch, fb, layer, q, k, v, **kw)
     _close(got, want)
-
-
-def _direct(q, kp, vp, r2t, row, pre, workspace=True, win=None, sinks=None):
-    """The C ABI's call for one request, with its workspace or without one (keys not split)."""
-    n, hq, d = q.shape
-    hkv, ints = kp.shape[1], ctypes.c_int32 * 1
-    lib = dk_lib.load()
-    new, alls = ints(n), ints(n + pre)
-    out = torch.full_like(q, float("nan"))
-    need = lib.dk_extend_workspace_bytes(1, new, alls, hq, hkv, d, win or 0) if workspace else 0
-    ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
-    s = dk_lib.DkExtendStrides(q.stride(0), d, kp.stride(0), d, vp.stride(0), d, out.stride(0), d)
-    rc = lib.dk_extend_attention(
-        q.data_ptr(), kp.data_ptr(), vp.data_ptr(), r2t.data_ptr(), r2t.stride(0), r2t.shape[0],
-        ints(row), new, alls, out.data_ptr(), None if ws is None else ws.data_ptr(), need, 1, n,
-        hq, hkv, d, kp.shape[0], 0 if q.dtype == torch.float16 else 1, dk_lib.DK_KV_SAME,
-        ctypes.byref(s), d ** -0.5, 1.0, 0.0, win or 0,
-        None if sinks is None else sinks.data_ptr(), torch.cuda.current_stream().cuda_stream)
-    dk_lib.check(rc, "dk_extend_attention")
-    return out, need
+    rows = fb.req_pool_indices.tolist()
+    outs = [_direct(q, pool.k_buffer[0], pool.v_buffer[0], fb.req_to_token_pool.req_to_token, rows,
+                    new, pre, w, win, kw.get("sinks"))
+            for w in (True, False, "short", "unaligned")]
+    splits = outs[0][1] > 0
+    assert splits == (new != [130])           # 130 keys are too few to split
+    for out, _ in outs:
+        _close(out.view_as(want), want)
+    assert torch.equal(outs[0][0].view_as(got), got)
+    assert all(torch.equal(out, outs[1][0]) for out, _ in outs[2 if splits else 0:])
 
 
 @pytest.mark.gpu
@@ -176,8 +190,8 @@ def test_a_key_that_draws_most_of_the_weight(dtype, d, new, pre, at, nats):
             mask, -math.inf), -1) @ vv[:, i // 4] for i in range(hq)], 1)
     rounding = float((want.to(dtype).double() - want).norm())
     for workspace in (True, False):
-        got, need = _direct(q, kp, vp, r2t, 0, pre, workspace)
-        assert (need > 0) == (workspace and n >= 512)          # both ways of the kernel
+        got, need = _direct(q, kp, vp, r2t, [0], [new], [pre], workspace)
+        assert (need > 0) == (n >= 512)                        # both ways of the kernel
         err = float((got.double() - want).norm())
         assert err <= 1.01 * rounding, (workspace, err / float(want.norm()), rounding / float(want.norm()))
 
