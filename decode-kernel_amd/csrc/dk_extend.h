@@ -16,12 +16,14 @@
 //     Each lane's accumulators all belong to its own query row, so rescaling is in-lane.
 //   * p enters as a sum of parts of the element type, 2 in fp16 and 3 in bf16 (ExtendParts).
 //     Scores, softmax, sums and accumulators are fp32.
-// Bound by the matrix cores: in bf16 at D = 128 the four MFMA streams (q.k and the 3 parts of
-// p) run at 1100 TFLOP/s of a large library product's 1267. 32/8/128 bf16, 2048 new of 8192
-// tokens: 437 us (551 TFLOP/s of attention; 371 us in fp16), the PyTorch path 6,200 us; 8
-// requests of 33-777 new tokens at D = 64, 57 us. 32 query rows per wavefront, so that two
-// wavefronts fit a SIMD (241 registers at D = 128) and one's softmax runs under the other's
-// MFMAs; 128 rows per workgroup keep the LDS reads at two thirds of the LDS rate.
+// Bound by the MFMAs and the softmax between them: in bf16 at D = 128 the four MFMA streams (q.k
+// and the 3 parts of p) run at 1100 TFLOP/s where a large library product reaches 1267, but a
+// SIMD is in an MFMA only 57 % of the time; the rest is exponentials and the split of the
+// weights, which the SIMD's other wavefront hides in part. 32/8/128, 2048 new of 8192 tokens,
+// back to back: bf16 441 us (546 TFLOP/s of attention), fp16 376; the PyTorch path 6,200 us. 8
+// requests of 33-777 new tokens over up to 500 at D = 64: 51-53 us (profiled, new inputs each
+// call). 32 query rows per wavefront, so that two wavefronts fit a SIMD (241 registers at D =
+// 128); 128 rows per workgroup keep the LDS reads at two thirds of the LDS rate.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -34,8 +36,11 @@ namespace dk {
 constexpr int kExtendRows = 128;      // query rows per workgroup
 constexpr int kExtendThreads = 256;
 // A call of fewer workgroups than fill the chip splits each query tile's keys over several, so
-// that about kExtendFill (two per CU) run, with at least kExtendSplitKeys keys each for the
-// longest request; fp32 partials and the decode merge kernel put them together. 32/8/128
+// that about kExtendFill run (two per CU, what a CU holds at D = 128, the only head_dim that the
+// figure was measured at; it holds three at D = 64 and one at D = 256), with at least
+// kExtendSplitKeys keys each for the longest request; one split for the whole call, so the
+// tiles of shorter requests get ranges without keys. fp32 partials and the decode merge kernel
+// put them together. 32/8/128
 // bf16, us, one workgroup per tile -> split: 16 new of 8,016 tokens 246 -> 21 (split 31), 8
 // requests of 16-64 new of 2,000-4,000 tokens 125 -> 64 (split 5); calls that fill the chip
 // keep one (2048 new of 8192 tokens 489 both).

@@ -1543,8 +1543,9 @@ __device__ __forceinline__ int cost_boundary(const Pass1Args& a, int base, int P
 // COST: the build whose range split charges sequence starts (a.seg_cost, ragged batches);
 // the other one splits equal pages and carries none of that code.
 // LONG: the build for ranges whose segments are long (long_segments in dk_api.hip): the pages
-// stream through stream_ring3 at up to 512 registers (its grid keeps one wavefront per SIMD
-// at most; at 256 the ring's loads are scheduled apart and it loses, 84.8 -> 90.8 us).
+// stream through stream_ring3. Its launch bounds ask for one wavefront per SIMD (its grid has
+// no more): the compiler then keeps the ring's loads together, in 207 and 215 registers (the
+// other build: 226 and 233); asked for two it schedules them apart and loses, 84.8 -> 90.8 us.
 template <class T, int D, int G, int NW, bool MFMA, bool KV8, int HP, bool COST = false,
           bool LONG = false>
 __global__ __launch_bounds__(NW * HP * 64, (LONG ? 1 : min_waves_per_simd<D, G, KV8>())) void dk_pass1_balanced(Pass1Args a) {
